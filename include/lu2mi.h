@@ -60,11 +60,12 @@ extern "C" {
                                      test that kernel alone);
                                      2: the same, with A taken as lower triangular (the U12
                                      product's form: entries above the diagonal are not read) */
-#define LU2MI_OPT_STRICT_SYNC 8   /* 1: the panel leaf and the back substitution publish their
-                                     cross-workgroup data with agent-scope release/acquire
-                                     (an L2 writeback and invalidate per publication); default
-                                     0: device-coherent stores completed in order (results
-                                     identical either way) */
+#define LU2MI_OPT_STRICT_SYNC 8   /* 1: the back substitution publishes its cross-workgroup
+                                     data with agent-scope release/acquire (an L2 writeback
+                                     and invalidate per publication); default 0:
+                                     device-coherent stores completed in order (results
+                                     identical either way).  The panel leaf needs neither:
+                                     each word it exchanges carries its own tag */
 #define LU2MI_OPT_WIDE16 9        /* 1: 16-bit trailing updates in 256 x 256 tiles (128 x 64 per
                                      wave) where they give every CU a workgroup; 0 (default):
                                      128 x 128 tiles (results identical either way) */

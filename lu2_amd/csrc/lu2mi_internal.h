@@ -84,7 +84,7 @@ struct lu2mi_ctx {
     int lookahead;         // factor panel i+1 on stream2 during block i's trailing update
     int trail_kernel;      // trailing-update tile: 1 direct-to-LDS FP64, 0 register-staged
     int dgemm_as_trailing; // lu2mi_dgemm_dev runs its product as a trailing update
-    int strict_sync;       // leaf and back substitution publish with release/acquire
+    int strict_sync;       // back substitution publishes with release/acquire
     int wide16;            // 16-bit updates in 256 x 256 tiles where they fill the device
     int backsub128;        // back substitution in 128-row blocks (64 otherwise)
     hipStream_t stream2;

@@ -38,7 +38,7 @@
 #include "lu2mi_internal.h"
 #include "lu2mi_dev.h"
 #include "lu2mi_gemm_tile.h"
-#include <limits.h>
+#include "lu2mi_leaf.h"
 #include <stdarg.h>
 #include <stdlib.h>
 #include <string.h>
@@ -83,463 +83,9 @@ __global__ __launch_bounds__(256) void diag_dominant_kernel(double *A, long lda,
     if (t == 0) A[r * lda + r] += (red[0] + red[1]) + (red[2] + red[3]);
 }
 
-// ---------------------------------------------------------------------------
-// Leaf factorization: persistent kernel over rows [c, n), W columns; all
-// workgroups are co-resident and meet at a grid barrier once per column.
-namespace {
-constexpr int SLOT_WORDS = 40;  // 3 header words + up to 32 row values; the last word is the sequence number
-constexpr int NTL = 256;        // threads per workgroup in the leaf kernel
-constexpr int LEAF_GMAX = 128;  // most workgroups a leaf launch may use
-
-__device__ __forceinline__ void st_relaxed(unsigned long long *p, unsigned long long v)
-{
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ unsigned long long ld_relaxed(unsigned long long *p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ unsigned long long dbits(double v) { return __double_as_longlong(v); }
-__device__ __forceinline__ double bitsd(unsigned long long v) { return __longlong_as_double(v); }
-// device-scope (coherent across XCDs) scalar loads and stores of a vector element
-__device__ __forceinline__ double ld_dev(const double *p)
-{
-    return bitsd(__hip_atomic_load((unsigned long long *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-}
-__device__ __forceinline__ float ld_dev(const float *p)
-{
-    return __uint_as_float(__hip_atomic_load((unsigned *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-}
-// device-scope loads through a buffer resource: same coherence as ld_dev but
-// without a wait after every load, so independent loads overlap
-__device__ __forceinline__ double ld_buf(__amdgpu_buffer_rsrc_t r, int byte_off, double)
-{
-    const unsigned int lo = __builtin_amdgcn_raw_buffer_load_b32(r, byte_off, 0, 16);
-    const unsigned int hi = __builtin_amdgcn_raw_buffer_load_b32(r, byte_off + 4, 0, 16);
-    return bitsd(((unsigned long long)hi << 32) | lo);
-}
-__device__ __forceinline__ float ld_buf(__amdgpu_buffer_rsrc_t r, int byte_off, float)
-{
-    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, byte_off, 0, 16));
-}
-__device__ __forceinline__ void st_dev(double *p, double v)
-{
-    __hip_atomic_store((unsigned long long *)p, dbits(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void st_dev(float *p, float v)
-{
-    __hip_atomic_store((unsigned *)p, __float_as_uint(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Publication of a sequence word (leaf slots, back-substitution frontier)
-// after the data it announces.  Every exchanged word is written and read with
-// device-coherent (agent-scope, sc1) accesses, so no cache maintenance is
-// needed, only completion order: the compiler barriers keep the data stores
-// ahead of the sequence store in program order and s_waitcnt vmcnt(0) makes
-// them complete before it is issued.  strict: an agent-scope release store
-// instead (on gfx950 it adds buffer_wbl2, an L2 writeback, per publication;
-// the matching acquire on the reader adds buffer_inv, an L2 invalidate).
-__device__ __forceinline__ void publish_seq(unsigned long long *p, unsigned long long v, int strict)
-{
-    if (strict) {
-        __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-    } else {
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        __builtin_amdgcn_s_waitcnt(0);
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-}
-// reader side, after the spin on a sequence word has seen the new value
-__device__ __forceinline__ void acquire_seq(int strict)
-{
-    if (strict) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    else __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-}
-
-// rank-1 update of one element: x - l * (u * s), with u*s rounded first (the
-// stored U value) and one fused multiply-subtract, written out so that every
-// copy of a row computes bit-identical values
-__device__ __forceinline__ double pending_update(double x, double l, double u, double s)
-{
-    return fma(-l, u * s, x);
-}
-__device__ __forceinline__ float pending_update(float x, float l, float u, float s)
-{
-    return fmaf(-l, u * s, x);
-}
-
-__device__ __forceinline__ bool better(double v, int r, double bv, int br)
-{
-    return (v > bv) || (v == bv && r < br);
-}
-}  // namespace
-
 // maximum that keeps a NaN (fmax drops it): a NaN solution must not pass as
 // a small residual
 __device__ __forceinline__ double nan_max(double a, double b) { return (a > b || a != a) ? a : b; }
-
-template <typename T>
-struct LeafArgs {
-    T *A;
-    long lda;
-    int n, c, i, compat;
-    int G;                        // number of workgroups (grid size)
-    int *piv;                     // global pivots, piv[j] for j in [c, c+W)
-    int *orig;                    // block-level origin row ids
-    T *invd;                      // 1/d per pivot row
-    int *pair_dst, *pair_src;     // 2W pairs for the panel row permutation
-    T *linv;                      // nb x nb inverse of D^-1 L11 (this leaf's block)
-    int ldl;
-    unsigned long long *slots;    // 2 * (G+1) * SLOT_WORDS, G <= LEAF_GMAX
-    unsigned long long seq_base;  // step sequence numbers seq_base+1 .. seq_base+W
-    int *err;
-    int strict;                   // release/acquire publication (publish_seq)
-};
-
-typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-
-// Per column step j (one grid-wide exchange):
-//   gather   every workgroup waits for the step's sequence number in each
-//            slot and copies all slots (candidate value, row, origins and
-//            the W values of the candidate row, plus the current row j) into
-//            LDS with device-scope buffer loads;
-//   reduce   each wavefront reduces the G candidates (largest |x|, lowest
-//            row on ties) -- identical result everywhere, no extra barrier;
-//   swap     the owners of rows j and p exchange rows, row j scaled by 1/d;
-//   column j+1 updated first, its candidate reduced in the workgroup and
-//            published (lookahead), then the other columns updated while
-//            the exchange is in flight.
-template <typename T, int W>
-struct LeafSmem {
-    T stage[NTL * (W + 1)];
-    unsigned long long xch[2][(LEAF_GMAX + 1) * (W + 3)];
-    double red_v[NTL / 64];
-    int red_r[NTL / 64];
-    int pivs[W];
-};
-
-// the leaf as workgroup bid of a.G (a stand-alone launch, or a phase of the
-// persistent sub-panel kernel)
-template <typename T, int W, int RPT>
-__device__ __forceinline__ void leaf_body(const LeafArgs<T> &a, const int bid, LeafSmem<T, W> &sm)
-{
-    constexpr int SW = W + 3;
-    T *const stage = sm.stage;
-    auto &xch = sm.xch;
-    double *const red_v = sm.red_v;
-    int *const red_r = sm.red_r;
-    int *const pivs = sm.pivs;
-
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int G = a.G;
-    const long TT = (long)G * NTL;
-    const int n = a.n, c = a.c;
-    T *__restrict__ A = a.A;
-    unsigned long long *const slots = a.slots;
-    const __amdgpu_buffer_rsrc_t srsrc =
-        __builtin_amdgcn_make_buffer_rsrc(slots, 0, (int)(2 * (G + 1) * SLOT_WORDS * 8), 0x00020000);
-
-    T row[RPT][W];
-    int lorig[RPT], borig[RPT], rq[RPT];
-
-    // coalesced load of the rows through LDS, one 256-row layer at a time
-#pragma clang loop unroll(full)
-    for (int q = 0; q < RPT; q++) {
-        const long base = (long)c + (long)bid * NTL + (long)q * TT;
-        rq[q] = (int)min((long)INT_MAX, base + t);
-        for (int e = t; e < NTL * W; e += NTL) {
-            const int rr = e / W, kk = e % W;
-            const long gr = base + rr;
-            stage[rr * (W + 1) + kk] = (gr < n) ? A[gr * a.lda + c + kk] : T(0);
-        }
-        __syncthreads();
-#pragma clang loop unroll(full)
-        for (int k = 0; k < W; k++) row[q][k] = stage[t * (W + 1) + k];
-        __syncthreads();
-        lorig[q] = rq[q];
-        borig[q] = (rq[q] < n) ? ((c == a.i) ? rq[q] : a.orig[rq[q]]) : -1;
-    }
-
-    // local candidate of column jc, workgroup reduction, publication of the
-    // slot (and of the current row by its owner in workgroup 0)
-    // pprev/sprev: the previous step's pivot slot and 1/d when that step's
-    // update of columns > jc is still pending (lookahead); the published
-    // values then carry it, computed exactly as the bulk update computes it
-    auto publish = [&](const int jc, const unsigned long long *pprev, const T sprev)
-                       __attribute__((always_inline)) {
-        const int j = c + jc;
-        const int par = jc & 1;
-        const unsigned long long seq = a.seq_base + (unsigned long long)jc + 1;
-        const bool odd_rule = a.compat && (jc & 1);
-        double bv = -1.0;
-        int br = INT_MAX;
-#pragma clang loop unroll(full)
-        for (int q = 0; q < RPT; q++) {
-            const int r = rq[q];
-            if (r >= j && r < n) {
-                const T xa = row[q][jc];
-                const T xb = row[q][jc > 0 ? jc - 1 : 0];
-                const double v = fabs((double)(odd_rule ? xb : xa));
-                if (v > bv) { bv = v; br = r; }
-            }
-        }
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            const double ov = __shfl_xor(bv, off);
-            const int orr = __shfl_xor(br, off);
-            if (better(ov, orr, bv, br)) { bv = ov; br = orr; }
-        }
-        if (lane == 0) { red_v[wave] = bv; red_r[wave] = br; }
-        __syncthreads();
-        double wv = red_v[0];
-        int wr = red_r[0];
-#pragma unroll
-        for (int w2 = 1; w2 < NTL / 64; w2++)
-            if (better(red_v[w2], red_r[w2], wv, wr)) { wv = red_v[w2]; wr = red_r[w2]; }
-        unsigned long long *sl = slots + ((long)par * (G + 1) + bid) * SLOT_WORDS;
-        auto value = [&](int q, int k) __attribute__((always_inline)) -> T {
-            if (pprev && k > jc) return pending_update(row[q][k], row[q][jc > 0 ? jc - 1 : 0], (T)bitsd(pprev[3 + k]), sprev);
-            return row[q][k];
-        };
-#pragma clang loop unroll(full)
-        for (int q = 0; q < RPT; q++)
-            if (rq[q] == wr && wr < n) {
-                st_relaxed(sl + 0, dbits(wv));
-                st_relaxed(sl + 1, (unsigned long long)(unsigned)wr);
-                st_relaxed(sl + 2, (unsigned long long)(unsigned)lorig[q] |
-                                       ((unsigned long long)(unsigned)borig[q] << 32));
-#pragma clang loop unroll(full)
-                for (int k = 0; k < W; k++) st_relaxed(sl + 3 + k, dbits((double)value(q, k)));
-                publish_seq(sl + SLOT_WORDS - 1, seq, a.strict);
-            }
-        if (wr >= n && t == 0) {
-            st_relaxed(sl + 0, dbits(-1.0));
-            st_relaxed(sl + 1, (unsigned long long)(unsigned)INT_MAX);
-            publish_seq(sl + SLOT_WORDS - 1, seq, a.strict);
-        }
-        if (bid == 0 && t == jc) {
-            unsigned long long *cs = slots + ((long)par * (G + 1) + G) * SLOT_WORDS;
-            st_relaxed(cs + 2, (unsigned long long)(unsigned)lorig[0] |
-                                   ((unsigned long long)(unsigned)borig[0] << 32));
-#pragma clang loop unroll(full)
-            for (int k = 0; k < W; k++) st_relaxed(cs + 3 + k, dbits((double)value(0, k)));
-            publish_seq(cs + SLOT_WORDS - 1, seq, a.strict);
-        }
-    };
-
-    publish(0, nullptr, T(0));
-#pragma clang loop unroll(full)
-    for (int jl = 0; jl < W; jl++) {
-        const int j = c + jl;
-        const int par = jl & 1;
-        const unsigned long long seq = a.seq_base + (unsigned long long)jl + 1;
-        unsigned long long *const xb = xch[par];
-        // ---- gather: thread g waits for slot g, then copies it to LDS
-        if (t <= G) {
-            unsigned long long *sl = slots + ((long)par * (G + 1) + t) * SLOT_WORDS;
-            unsigned long spins = 0;
-            while (ld_relaxed(sl + SLOT_WORDS - 1) != seq) {
-                __builtin_amdgcn_s_sleep(1);
-                if (((++spins) & 1023) == 0) {
-                    if (__hip_atomic_load(a.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) break;
-                    if (spins > (1UL << 25)) {
-                        __hip_atomic_store(a.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        break;
-                    }
-                }
-            }
-            acquire_seq(a.strict);
-            const int boff = (int)(((long)par * (G + 1) + t) * SLOT_WORDS * 8);
-#pragma clang loop unroll(full)
-            for (int k = 0; k < SW; k++) {
-                const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(srsrc, boff + 8 * k, 0, 16);
-                xb[t * SW + k] = ((unsigned long long)v.y << 32) | v.x;
-            }
-        }
-        __syncthreads();
-        // ---- every wavefront reduces the G candidates (same result everywhere)
-        double bv = -1.0;
-        int br = INT_MAX, bg = -1;
-        for (int g2 = lane; g2 < G; g2 += 64) {
-            const double v = bitsd(xb[g2 * SW + 0]);
-            const int r = (int)(unsigned)xb[g2 * SW + 1];
-            if (better(v, r, bv, br)) { bv = v; br = r; bg = g2; }
-        }
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            const double ov = __shfl_xor(bv, off);
-            const int orr = __shfl_xor(br, off);
-            const int og = __shfl_xor(bg, off);
-            if (better(ov, orr, bv, br)) { bv = ov; br = orr; bg = og; }
-        }
-        // no comparable candidate (every |x| is NaN): pivot on the current
-        // row, as BLAS idamax returns the first index for NaN input
-        const bool none = (br < j || br >= n || bg < 0);
-        const int p = none ? j : br;
-        const unsigned long long *pslot = xb + (none ? G : bg) * SW;
-        const unsigned long long *cslot = xb + G * SW;
-        const int p_lorig = (int)(unsigned)(pslot[2] & 0xffffffffULL), p_borig = (int)(unsigned)(pslot[2] >> 32);
-        const int c_lorig = (int)(unsigned)(cslot[2] & 0xffffffffULL), c_borig = (int)(unsigned)(cslot[2] >> 32);
-#define PIVROW(k) ((T)bitsd(pslot[3 + (k)]))
-#define CURROW(k) ((T)bitsd(cslot[3 + (k)]))
-        const T d = PIVROW(jl);
-        const T s = T(1) / d;
-        // ---- swap rows j and p; row j becomes the pivot row scaled by 1/d
-#pragma clang loop unroll(full)
-        for (int q = 0; q < RPT; q++) {
-            const int r = rq[q];
-            if (r == j) {
-#pragma clang loop unroll(full)
-                for (int k = 0; k < W; k++) row[q][k] = (k == jl) ? d : PIVROW(k) * s;
-                lorig[q] = p_lorig;
-                borig[q] = p_borig;
-            } else if (r == p) {
-#pragma clang loop unroll(full)
-                for (int k = 0; k < W; k++) row[q][k] = CURROW(k);
-                lorig[q] = c_lorig;
-                borig[q] = c_borig;
-            }
-        }
-        // ---- column j+1 first, then publish its candidate (lookahead)
-        if (jl + 1 < W) {
-#pragma clang loop unroll(full)
-            for (int q = 0; q < RPT; q++) {
-                const int r = rq[q];
-                if (r > j && r < n) {
-                    T &x1 = row[q][jl + 1 < W ? jl + 1 : 0];
-                    x1 = pending_update(x1, row[q][jl], PIVROW(jl + 1 < W ? jl + 1 : 0), s);
-                }
-            }
-            publish(jl + 1 < W ? jl + 1 : 0, pslot, s);
-        }
-        // ---- the remaining columns while the exchange is in flight
-#pragma clang loop unroll(full)
-        for (int q = 0; q < RPT; q++) {
-            const int r = rq[q];
-            if (r > j && r < n) {
-                const T l = row[q][jl];
-#pragma clang loop unroll(full)
-                for (int k = jl + 2; k < W; k++) row[q][k] = pending_update(row[q][k], l, PIVROW(k), s);
-            }
-        }
-        if (t == 0) {
-            pivs[jl] = p;
-            if (bid == 0) {
-                a.piv[j] = p;
-                a.invd[j] = s;
-            }
-        }
-#undef PIVROW
-#undef CURROW
-    }
-    __syncthreads();
-
-    // ---- write back rows (coalesced through LDS), origins and row pairs
-#pragma clang loop unroll(full)
-    for (int q = 0; q < RPT; q++) {
-        const long base = (long)c + (long)bid * NTL + (long)q * TT;
-#pragma clang loop unroll(full)
-        for (int k = 0; k < W; k++) stage[t * (W + 1) + k] = row[q][k];
-        __syncthreads();
-        for (int e = t; e < NTL * W; e += NTL) {
-            const int rr = e / W, kk = e % W;
-            const long gr = base + rr;
-            if (gr < n) A[gr * a.lda + c + kk] = stage[rr * (W + 1) + kk];
-        }
-        __syncthreads();
-        const int r = rq[q];
-        if (r < n) {
-            a.orig[r] = borig[q];
-#pragma clang loop unroll(full)
-            for (int k = 0; k < W; k++)
-                if (pivs[k] == r) {
-                    a.pair_dst[W + k] = r;
-                    a.pair_src[W + k] = lorig[q];
-                }
-        }
-    }
-    if (bid == 0) {
-        if (t < W) {
-            a.pair_dst[t] = c + t;
-            a.pair_src[t] = lorig[0];
-            // leaf block of the inverse of the unit-lower D^-1 L11
-#pragma clang loop unroll(full)
-            for (int k = 0; k < W; k++) stage[t * (W + 1) + k] = row[0][k];
-        }
-        __syncthreads();
-        if (t < W) {
-            T x[W];
-#pragma clang loop unroll(full)
-            for (int r = 0; r < W; r++) {
-                if (r < t) x[r] = T(0);
-                else if (r == t) x[r] = T(1);
-                else {
-                    T acc = T(0);
-#pragma clang loop unroll(full)
-                    for (int k = 0; k < r; k++)
-                        if (k >= t) acc += stage[r * (W + 1) + k] * x[k];
-                    x[r] = -acc;
-                }
-            }
-            const long off = (long)(c - a.i);
-#pragma clang loop unroll(full)
-            for (int r = 0; r < W; r++) a.linv[(off + r) * a.ldl + off + t] = x[r];
-        }
-    }
-}
-
-template <typename T, int W, int RPT>
-__global__ __launch_bounds__(NTL) void leaf_kernel(LeafArgs<T> a)
-{
-    __shared__ LeafSmem<T, W> sm;
-    leaf_body<T, W, RPT>(a, blockIdx.x, sm);
-}
-
-// ---------------------------------------------------------------------------
-// Row permutation of a column range: all sources of a column strip are read
-// into LDS before any destination is written, so in-place permutations are
-// safe.  Destinations in [d0, d1) are scaled by invd[dst] on columns < sce;
-// destinations in [w0, w1) are written to the staging buffer instead.
-template <typename T>
-struct PermArgs {
-    T *A;
-    long lda;
-    const int *dst, *src;
-    int np;
-    int c0, c1, k0, k1;   // columns [c0, c1) except [k0, k1)
-    int sce;              // scale columns < sce
-    int d0, d1;
-    const T *invd;
-    T *W;
-    long ldw;
-    int w0, w1;
-    int sw;               // strip width
-};
-
-template <typename T>
-__device__ __forceinline__ void rowperm_strip(const PermArgs<T> &a, const int strip, T *buf)
-{
-    const int cs = a.c0 + strip * a.sw;
-    const int total = a.np * a.sw;
-    for (int e = threadIdx.x; e < total; e += 256) {
-        const int pr = e / a.sw, cc = e % a.sw;
-        const int col = cs + cc;
-        if (col < a.c1 && (col < a.k0 || col >= a.k1)) buf[e] = a.A[(long)a.src[pr] * a.lda + col];
-    }
-    __syncthreads();
-    for (int e = threadIdx.x; e < total; e += 256) {
-        const int pr = e / a.sw, cc = e % a.sw;
-        const int col = cs + cc;
-        if (col < a.c1 && (col < a.k0 || col >= a.k1)) {
-            const int d = a.dst[pr];
-            T v = buf[e];
-            if (d >= a.d0 && d < a.d1 && col < a.sce) v *= a.invd[d];
-            if (d >= a.w0 && d < a.w1) a.W[(long)(d - a.w0) * a.ldw + (col - a.c0)] = v;
-            else a.A[(long)d * a.lda + col] = v;
-        }
-    }
-}
 
 template <typename T>
 __global__ __launch_bounds__(256) void rowperm_kernel(PermArgs<T> a)
@@ -602,163 +148,6 @@ __global__ void scale_copy_kernel(const T *A, long lda, int r0, int c0, int h, i
         W[e] = A[(long)(r0 + r) * lda + c0 + col] * invd[r0 + r];
     }
 }
-
-// ---------------------------------------------------------------------------
-// Persistent sub-panel: one launch factors w columns [c, c+w) of the block's
-// panel (w a power of two <= SUB_WMAX, 16-column leaves): every leaf, its row
-// swaps over the panel's other columns, and every recursion node inside the
-// sub-panel (1/d scaling and staging, explicit-inverse TRSM, update of the
-// rows below, off-diagonal block of the inverse), in the order of the
-// recursion of lu2.c:1187-1235, separated by grid barriers instead of kernel
-// boundaries.  The steps run the same device code as the separate launches
-// (leaf body, row-swap strip, GEMM tile), so the factors are bit-identical;
-// the difference is one dispatch instead of about seven per leaf, which is
-// what a panel factored beside the trailing update waits on.
-constexpr int SUB_W = 16;       // leaf width inside the sub-panel kernel
-constexpr int SUB_WMAX = 256;   // widest sub-panel
-constexpr int SUB_SWMAX = 128;  // widest row-swap strip (LDS: 2*SUB_W pairs x strip)
-constexpr size_t SLOTS_BYTES = sizeof(unsigned long long) * 2 * (size_t)(1024 + 1) * SLOT_WORDS;
-
-template <typename T>
-struct SubArgs {
-    LeafArgs<T> leaf;            // first leaf: c = sub-panel start, seq_base of its first column
-    int nb, w, sw;               // block size, sub-panel width, row-swap strip width
-    T *wbuf, *tmp;               // h x h staging of the scaled rows; h x h product scratch
-    unsigned long long *gbar;    // grid barrier arrivals (monotonic within a factorization)
-    unsigned long long gbar_base;
-};
-
-// Barrier over the G co-resident workgroups: arrivals counted on one word,
-// agent-scope fences on both sides so that every step's global writes (on
-// any XCD) are visible to the next step.  Bounded: a timeout raises *err and
-// lets every wave run to the end of the kernel.
-__device__ __forceinline__ void grid_sync(unsigned long long *ctr, unsigned long long target, int *err)
-{
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        __threadfence();
-        __hip_atomic_fetch_add(ctr, 1ULL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        unsigned long spins = 0;
-        while (__hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
-            __builtin_amdgcn_s_sleep(1);
-            if (((++spins) & 1023) == 0) {
-                if (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) break;
-                if (spins > (1UL << 25)) {
-                    __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    break;
-                }
-            }
-        }
-        __threadfence();
-    }
-    __syncthreads();
-}
-
-// C = alpha A B + beta C over the G workgroups in 64x64 tiles, each with the
-// K range of the stand-alone GEMM's 128x128 tile that contains it
-template <typename T, int EPI>
-__device__ __forceinline__ void gemm_steps(int M, int N, int K, double alpha, const T *A, long lda, const T *B,
-                                           long ldb, double beta, T *C, long ldc, int a_lower, int bid, int G,
-                                           lu2mi_gemm::Tile64Smem<T> &ts)
-{
-    using namespace lu2mi_gemm;
-    GemmDesc g;
-    g.M = M; g.N = N; g.K = K; g.alpha = alpha; g.beta = beta;
-    g.A = A; g.lda = lda; g.B = B; g.ldb = ldb; g.C = C; g.ldc = ldc; g.a_lower = a_lower;
-    const int tiles_m = (M + BT64 - 1) / BT64, tiles_n = (N + BT64 - 1) / BT64;
-    const int total = (M > 0 && N > 0) ? tiles_m * tiles_n : 0;
-    for (int tile = bid; tile < total; tile += G) {
-        const int m0 = (tile / tiles_n) * BT64, n0 = (tile % tiles_n) * BT64;
-        const int Kt = a_lower ? min(K, (m0 & ~(BM - 1)) + BM) : K;
-        const bool interior = (m0 + BT64 <= M) && (n0 + BT64 <= N) && (Kt % Mfma<T>::BK == 0);
-        if (interior) gemm_tile64<T, false, EPI>(g, A, B, C, m0, n0, Kt, ts);
-        else gemm_tile64<T, true, EPI>(g, A, B, C, m0, n0, Kt, ts);
-        __syncthreads();   // the next tile restages the same LDS
-    }
-}
-
-template <typename T, int RPT>
-__global__ __launch_bounds__(NTL, 2) void subpanel_kernel(SubArgs<T> s)
-{
-    using namespace lu2mi_gemm;
-    constexpr int W = SUB_W;
-    __shared__ union {
-        LeafSmem<T, W> leaf;
-        Tile64Smem<T> tile;
-        T perm[2 * W * SUB_SWMAX];
-    } sm;
-    const int bid = blockIdx.x, G = s.leaf.G;
-    const int i = s.leaf.i, n = s.leaf.n, c0 = s.leaf.c, nb = s.nb, L = s.w / W;
-    const long lda = s.leaf.lda;
-    const int ldl = s.leaf.ldl;
-    T *const A = s.leaf.A;
-    T *const linv = s.leaf.linv;
-    unsigned long long target = s.gbar_base;
-    auto sync = [&]() __attribute__((always_inline)) {
-        target += (unsigned long long)G;
-        grid_sync(s.gbar, target, s.leaf.err);
-    };
-    // node (cn, 2h) after its left half: rows [cn, cn+h) of the right half
-    // scaled by 1/d and staged, X = inv(D^-1 L11) * staged rows, then the
-    // rows below (host path: Factor::panel)
-    auto node_mid = [&](const int cn, const int h) __attribute__((always_inline)) {
-        const long off = cn - i;
-        for (long e = (long)bid * NTL + threadIdx.x; e < (long)h * h; e += (long)G * NTL) {
-            const int r = (int)(e / h), col = (int)(e % h);
-            s.wbuf[e] = A[(long)(cn + r) * lda + cn + h + col] * s.leaf.invd[cn + r];
-        }
-        sync();
-        gemm_steps<T, EPI_SET>(h, h, h, 1.0, linv + off * ldl + off, ldl, s.wbuf, h, 0.0,
-                               A + (long)cn * lda + cn + h, lda, 1, bid, G, sm.tile);
-        sync();
-        gemm_steps<T, EPI_SUB>(n - cn - h, h, h, -1.0, A + (long)(cn + h) * lda + cn, lda,
-                               A + (long)cn * lda + cn + h, lda, 1.0, A + (long)(cn + h) * lda + cn + h, lda, 0,
-                               bid, G, sm.tile);
-        sync();
-    };
-    // node (cn, 2h) after its right half: X21 = -inv22 * L21 * inv11
-    auto node_end = [&](const int cn, const int h) __attribute__((always_inline)) {
-        const long off = cn - i;
-        gemm_steps<T, EPI_SET>(h, h, h, 1.0, A + (long)(cn + h) * lda + cn, lda, linv + off * ldl + off, ldl, 0.0,
-                               s.tmp, h, 0, bid, G, sm.tile);
-        sync();
-        gemm_steps<T, EPI_GENERAL>(h, h, h, -1.0, linv + (off + h) * ldl + off + h, ldl, s.tmp, h, 0.0,
-                                   linv + (off + h) * ldl + off, ldl, 1, bid, G, sm.tile);
-        sync();
-    };
-    // post-order walk: before leaf k the nodes whose right half ended at
-    // leaf k-1 (deepest first) get their inverse block, then the node whose
-    // left half ended there gets its right half updated
-    for (int k = 0; k <= L; k++) {
-        if (k > 0) {
-            const int tz = __builtin_ctz(k);
-            for (int lv = 1; lv <= tz; lv++) node_end(c0 + (k - (1 << lv)) * W, W << (lv - 1));
-            if (k == L) break;
-            node_mid(c0 + (k - (1 << tz)) * W, W << tz);
-        }
-        LeafArgs<T> la = s.leaf;
-        la.c = c0 + k * W;
-        la.seq_base = s.leaf.seq_base + (unsigned long long)k * W;
-        leaf_body<T, W, RPT>(la, bid, sm.leaf);
-        sync();
-        // the leaf's swaps on the panel's other columns; its diagonal rows'
-        // L part (columns left of the leaf) scaled by 1/d
-        PermArgs<T> p;
-        p.A = A; p.lda = lda; p.dst = la.pair_dst; p.src = la.pair_src; p.np = 2 * W;
-        p.c0 = i; p.c1 = i + nb; p.k0 = la.c; p.k1 = la.c + W; p.sce = la.c; p.d0 = la.c; p.d1 = la.c + W;
-        p.invd = la.invd; p.W = nullptr; p.ldw = 0; p.w0 = 0; p.w1 = 0; p.sw = s.sw;
-        const int strips = (nb + s.sw - 1) / s.sw;
-        for (int st = bid; st < strips; st += G) {
-            rowperm_strip<T>(p, st, sm.perm);
-            __syncthreads();
-        }
-        sync();
-    }
-}
-
-// grid barriers one sub-panel launch of L leaves passes: two per leaf, three
-// per node before its right half, two per node after it
-__host__ __device__ constexpr int sub_barriers(int L) { return 2 * L + 5 * (L - 1); }
 
 // ---------------------------------------------------------------------------
 // Recursion nodes of half-width h <= 64, one workgroup (one 64x64 tile) per
@@ -840,17 +229,6 @@ __global__ void copy_col_kernel(const T *A, long lda, int n, int col, T *x)
 // entry.  TF is the factor's element type, TX the vector's (FP64 for
 // refinement).
 constexpr int BSB = 64;
-
-__device__ __forceinline__ double lane_bcast(double v, int l)
-{
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane((int)b, l), hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-__device__ __forceinline__ float lane_bcast(float v, int l)
-{
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
-}
 
 template <typename TF, typename TX, int BS>
 __global__ __launch_bounds__(BS * 4) void backsub_kernel(const TF *__restrict__ A, long lda, int n, TX *x,
@@ -1279,6 +657,10 @@ struct Factor {
         if (W == 32 && rpt > 2) rpt = 2;
         if (W == 16 && rpt > 4) rpt = 4;
         if (rpt == 3) rpt = 4;
+        // as many rows as one workgroup's registers hold: no exchange through
+        // memory at all
+        const int rmax = (W == 16) ? 4 : 2;
+        if (R <= NTL * rmax) rpt = (R <= NTL) ? 1 : (R <= 2 * NTL) ? 2 : 4;
         const int G = (R + NTL * rpt - 1) / (NTL * rpt);
         if (G > LEAF_GMAX) {
             lu2mi_set_error_msg("leaf: %d rows need %d workgroups (> %d)", R, G, LEAF_GMAX);
@@ -1290,7 +672,7 @@ struct Factor {
         la.pair_dst = pairs; la.pair_src = pairs + 2 * W;
         la.linv = linv; la.ldl = nb;
         la.slots = (unsigned long long *)ctx->d_slots;
-        la.seq_base = ctx->bar_count; la.err = ctx->d_err; la.strict = ctx->strict_sync;
+        la.seq_base = ctx->bar_count; la.err = ctx->d_err;
         void *args[] = {&la};
         const void *fn = nullptr;
         if (W == 32) fn = (rpt == 1) ? (const void *)leaf_kernel<T, 32, 1> : (const void *)leaf_kernel<T, 32, 2>;
@@ -1394,7 +776,7 @@ struct Factor {
         la.pair_dst = pairs; la.pair_src = pairs + 2 * SUB_W;
         la.linv = linv; la.ldl = nb;
         la.slots = (unsigned long long *)ctx->d_slots;
-        la.seq_base = ctx->bar_count; la.err = ctx->d_err; la.strict = ctx->strict_sync;
+        la.seq_base = ctx->bar_count; la.err = ctx->d_err;
         sa.nb = nb; sa.w = w;
         // strips of at least 64 bytes per row, about one per workgroup
         const int seg = 64 / (int)sizeof(T);
