@@ -25,6 +25,7 @@ template <typename T, int EPI>
 __global__ __launch_bounds__(NT) void gemm64_kernel(GemmDesc g, int tiles_m, int tiles_n)
 {
     __shared__ Tile64Smem<T> sm;
+    __builtin_amdgcn_s_setprio(3);   // the panel's products, beside a trailing update
     const int m0 = (blockIdx.x / tiles_n) * BT64, n0 = (blockIdx.x % tiles_n) * BT64;
     const long bz = blockIdx.y;
     const T *A = (const T *)g.A + bz * g.sA;

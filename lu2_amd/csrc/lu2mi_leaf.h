@@ -595,6 +595,7 @@ template <typename T, int W, int RPT>
 __global__ __launch_bounds__(NTL, W == 16 ? 2 : 1) void leaf_kernel(LeafArgs<T> a)
 {
     __shared__ LeafSmem<T, W> sm;
+    __builtin_amdgcn_s_setprio(3);   // ahead of the trailing update's waves beside it, as all of the panel's kernels
     leaf_body<T, W, RPT>(a, blockIdx.x, sm);
 }
 

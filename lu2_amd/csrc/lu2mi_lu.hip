@@ -91,6 +91,7 @@ template <typename T>
 __global__ __launch_bounds__(256) void rowperm_kernel(PermArgs<T> a)
 {
     extern __shared__ unsigned char smem_raw[];
+    __builtin_amdgcn_s_setprio(3);
     rowperm_strip<T>(a, blockIdx.x, (T *)smem_raw);
 }
 
@@ -161,6 +162,7 @@ __global__ __launch_bounds__(256) void node_trsm64_kernel(T *A, long lda, int c,
 {
     using namespace lu2mi_gemm;
     __shared__ Tile64Smem<T> sm;
+    __builtin_amdgcn_s_setprio(3);
     GemmDesc g;
     g.M = h; g.N = h; g.K = h; g.alpha = 1.0; g.beta = 0.0;
     g.lda = ldl; g.ldb = lda; g.ldc = lda; g.a_lower = 1;
@@ -176,6 +178,7 @@ __global__ __launch_bounds__(256) void node_inv64_kernel(const T *A, long lda, i
 {
     using namespace lu2mi_gemm;
     __shared__ Tile64Smem<T> sm;
+    __builtin_amdgcn_s_setprio(3);
     GemmDesc g;
     g.M = h; g.N = h; g.K = h; g.alpha = 1.0; g.beta = 0.0;
     g.lda = lda; g.ldb = ldl; g.ldc = h; g.a_lower = 0;
@@ -960,6 +963,17 @@ struct Factor {
             if (la) {
                 LU2MI_TRY(trailing(i, i + nb, nb));                    // the next panel's columns
                 LU2MI_CHECK(hipEventRecord(ctx->ev_next, s1));
+                // the rest of block i, b included: staging rows from column nb
+                // of w on, so that w keeps the layout of the unsplit product.
+                // Queued before the panel: a panel is some two hundred
+                // launches (n = 32768, nb = 512), and from the middle of the
+                // factorization on the device had run them all when the last
+                // was queued, with this stream idle beside it: 521 -> 512 ms,
+                // n = 49152, nb = 1024 1405 -> 1384 ms, with the panel's
+                // kernels at a higher wave priority.
+                LU2MI_TRY(block_perm(i, i + 2 * nb, n + 1, wbuf + nb, ldw));
+                LU2MI_TRY(u12(i, i + 2 * nb, ncols - nb, wbuf + nb, ldw));
+                LU2MI_TRY(trailing(i, i + 2 * nb, ncols - nb));
                 LU2MI_CHECK(hipStreamWaitEvent(ctx->stream2, ctx->ev_next, 0));
                 ctx->stream = ctx->stream2;                           // panel(i+nb) on the second stream
                 const int prc = start_panel(i + nb);
@@ -967,12 +981,6 @@ struct Factor {
                 LU2MI_TRY(prc);
                 LU2MI_CHECK(hipEventRecord(ctx->ev_panel, ctx->stream2));
                 panel_pending = true;
-                // the rest of block i, b included: staging rows from column nb
-                // of w on, so that w keeps the layout of the unsplit product
-                set_block(i);
-                LU2MI_TRY(block_perm(i, i + 2 * nb, n + 1, wbuf + nb, ldw));
-                LU2MI_TRY(u12(i, i + 2 * nb, ncols - nb, wbuf + nb, ldw));
-                LU2MI_TRY(trailing(i, i + 2 * nb, ncols - nb));
             } else {
                 LU2MI_TRY(trailing(i, i + nb, ncols));
                 LU2MI_TRY(start_panel(i + nb));
