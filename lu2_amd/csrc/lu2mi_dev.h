@@ -50,6 +50,7 @@ template <typename T> struct Mfma;
 template <> struct Mfma<double> {
     typedef d4_t acc_t;
     typedef double2 vec_t;   // 16 bytes
+    typedef double uvec_t __attribute__((ext_vector_type(2), aligned(8)));   // the same from any element on
     static constexpr int BK = 16, EPV = 2;
     static __device__ __forceinline__ acc_t step(double a, double b, acc_t c)
     {
@@ -60,6 +61,7 @@ template <> struct Mfma<double> {
 template <> struct Mfma<float> {
     typedef f4_t acc_t;
     typedef float4 vec_t;
+    typedef float uvec_t __attribute__((ext_vector_type(4), aligned(4)));
     static constexpr int BK = 32, EPV = 4;
     static __device__ __forceinline__ acc_t step(float a, float b, acc_t c)
     {

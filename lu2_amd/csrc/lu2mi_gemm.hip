@@ -21,7 +21,7 @@ using namespace lu2mi_gemm;
 // padding and spread over more workgroups; every element keeps the K range
 // of the 128x128 tile that contains it, so the results are the 128x128
 // kernel's bits.
-template <typename T, int EPI>
+template <typename T, int EPI, bool VEC, bool DORD = false>
 __global__ __launch_bounds__(NT) void gemm64_kernel(GemmDesc g, int tiles_m, int tiles_n)
 {
     __shared__ Tile64Smem<T> sm;
@@ -33,8 +33,8 @@ __global__ __launch_bounds__(NT) void gemm64_kernel(GemmDesc g, int tiles_m, int
     T *C = (T *)g.C + bz * g.sC;
     const int K = g.a_lower ? min(g.K, (m0 & ~(BM - 1)) + BM) : g.K;
     const bool interior = (m0 + BT64 <= g.M) && (n0 + BT64 <= g.N) && (K % Mfma<T>::BK == 0);
-    if (interior) gemm_tile64<T, false, EPI>(g, A, B, C, m0, n0, K, sm);
-    else gemm_tile64<T, true, EPI>(g, A, B, C, m0, n0, K, sm);
+    if (interior) gemm_tile64<T, false, EPI, VEC, DORD>(g, A, B, C, m0, n0, K, sm);
+    else gemm_tile64<T, true, EPI, VEC, DORD>(g, A, B, C, m0, n0, K, sm);
 }
 
 template <typename T, bool VEC, int EPI, int TAG>
@@ -158,7 +158,13 @@ static int launch_gemm(const GemmDesc &g, hipStream_t s)
         lu2mi_set_error_msg("gemm: grid too large");
         return LU2MI_ERR_ARG;
     }
-    // 16-byte vector loads need 16-byte aligned rows of A and B
+    // 16-byte aligned rows of A and B; others (an odd row stride or first
+    // column) run the 64x64 tiles with unaligned 16-byte loads, in one general
+    // form (element loads with bounds checks in 128x128 tiles before: at an odd
+    // stride 700 x 900 x 300 80 -> 40 us, 40 x 8000 x 100 43 -> 28 us,
+    // 3000 x 3000 x 1000 473 -> 392 us), and above the 64x64 tiles' sizes the
+    // 128x128 tiles with element loads (6001 x 6001 x 513 806 us, 822 with
+    // unaligned ones)
     constexpr long EPV = Mfma<T>::EPV;
     const bool vec = aligned16(g.A) && aligned16(g.B) && (g.lda % EPV == 0) && (g.ldb % EPV == 0) &&
                      (g.sA % EPV == 0) && (g.sB % EPV == 0);
@@ -175,22 +181,47 @@ static int launch_gemm(const GemmDesc &g, hipStream_t s)
         LU2MI_CHECK(hipDeviceGetAttribute(&num_cu, hipDeviceAttributeMultiprocessorCount, dev));
     }
     const bool underfilled = total * g.batch < 8L * num_cu;
-    if (vec && g.tag == 0 && (g.M <= BT64 || g.N <= BT64 || underfilled)) {
+    const bool direct = sizeof(T) == 8 && g.tag == 1 && vec && g.batch == 1 && aligned16(g.C) && g.ldc % 2 == 0;
+    // Trailing updates and U12 products with less than one 128x128 tile per CU
+    // (small matrices, and the next panel's columns of larger ones): 64x64
+    // tiles here too, in the K order of the tile they stand for (same bits).
+    // n = 512 nb = 64 2.40 -> 2.20 ms, n = 2048 nb = 256 10.0 -> 9.55 ms (a
+    // 128x128 U12 product of 256 columns there took 65 us), n = 9984 nb = 256
+    // 62.5 -> 59.9 ms.
+    if (vec && g.tag != 0 && g.batch == 1 && total < num_cu && (sizeof(T) == 4 || direct || g.tag == 2) &&
+        (g.a_lower ? epi == EPI_SET : epi == EPI_SUB)) {
+        const int tm64 = (g.M + BT64 - 1) / BT64, tn64 = (g.N + BT64 - 1) / BT64;
+        dim3 grid64((unsigned)(tm64 * tn64)), block64(NT);
+        constexpr bool DO = sizeof(T) == 8;
+        if (epi == EPI_SET && direct)
+            hipLaunchKernelGGL((gemm64_kernel<T, EPI_SET, true, DO>), grid64, block64, 0, s, g, tm64, tn64);
+        else if (epi == EPI_SET)
+            hipLaunchKernelGGL((gemm64_kernel<T, EPI_SET, true>), grid64, block64, 0, s, g, tm64, tn64);
+        else if (direct)
+            hipLaunchKernelGGL((gemm64_kernel<T, EPI_SUB, true, DO>), grid64, block64, 0, s, g, tm64, tn64);
+        else
+            hipLaunchKernelGGL((gemm64_kernel<T, EPI_SUB, true>), grid64, block64, 0, s, g, tm64, tn64);
+        LU2MI_CHECK(hipGetLastError());
+        return LU2MI_OK;
+    }
+    if (g.tag == 0 && (g.M <= BT64 || g.N <= BT64 || underfilled)) {
         const int tm64 = (g.M + BT64 - 1) / BT64, tn64 = (g.N + BT64 - 1) / BT64;
         dim3 grid64((unsigned)(tm64 * tn64), (unsigned)g.batch), block64(NT);
-        if (epi == EPI_SUB)
-            hipLaunchKernelGGL((gemm64_kernel<T, EPI_SUB>), grid64, block64, 0, s, g, tm64, tn64);
+        if (!vec)
+            hipLaunchKernelGGL((gemm64_kernel<T, EPI_GENERAL, false>), grid64, block64, 0, s, g, tm64, tn64);
+        else if (epi == EPI_SUB)
+            hipLaunchKernelGGL((gemm64_kernel<T, EPI_SUB, true>), grid64, block64, 0, s, g, tm64, tn64);
         else if (epi == EPI_SET)
-            hipLaunchKernelGGL((gemm64_kernel<T, EPI_SET>), grid64, block64, 0, s, g, tm64, tn64);
+            hipLaunchKernelGGL((gemm64_kernel<T, EPI_SET, true>), grid64, block64, 0, s, g, tm64, tn64);
         else
-            hipLaunchKernelGGL((gemm64_kernel<T, EPI_GENERAL>), grid64, block64, 0, s, g, tm64, tn64);
+            hipLaunchKernelGGL((gemm64_kernel<T, EPI_GENERAL, true>), grid64, block64, 0, s, g, tm64, tn64);
         LU2MI_CHECK(hipGetLastError());
         return LU2MI_OK;
     }
     if (g.a_lower && epi == EPI_SET && vec && g.batch == 1) {
         // the U12 product: pairs of row tiles per workgroup
         dim3 gridp((unsigned)((long)((tiles_m + 1) / 2) * tiles_n)), blockp(NT);
-        if (sizeof(T) == 8 && g.tag == 1 && aligned16(g.C) && g.ldc % 2 == 0)
+        if (direct)
             hipLaunchKernelGGL(gemm2_lower_kernel, gridp, blockp, 0, s, g, tiles_m, tiles_n);
         else
             hipLaunchKernelGGL(gemm_lower_kernel<T>, gridp, blockp, 0, s, g, tiles_m, tiles_n);
@@ -198,8 +229,7 @@ static int launch_gemm(const GemmDesc &g, hipStream_t s)
         return LU2MI_OK;
     }
     dim3 grid((unsigned)total, (unsigned)g.batch), block(NT);
-    if (sizeof(T) == 8 && g.tag == 1 && epi == EPI_SUB && vec && g.batch == 1 &&
-        !g.a_lower && aligned16(g.C) && g.ldc % 2 == 0) {
+    if (direct && epi == EPI_SUB && !g.a_lower) {
         hipLaunchKernelGGL(gemm2_kernel<EPI_SUB>, grid, block, 0, s, g, tiles_m, tiles_n);
         LU2MI_CHECK(hipGetLastError());
         return LU2MI_OK;

@@ -23,6 +23,28 @@ constexpr int BM = 128, BN = 128, NT = 256;
 //                 EPI_SET      C = acc            (alpha = 1, beta = 0: the TRSM products)
 enum { EPI_GENERAL = 0, EPI_SUB = 1, EPI_SET = 2 };
 
+// Place of a stage's k in LDS.  DORD (FP64): the K order of the direct-to-LDS
+// tile (below), whose MFMA step s takes k = 4q + s from lane group q, here
+// found at place 4s + q; the results are then that tile's bits.
+template <bool DORD>
+__device__ __forceinline__ constexpr int k_place(int k)
+{
+    return DORD ? ((k & 3) << 2) | (k >> 2) : k;
+}
+
+// 16 bytes of a row; VEC: 16-byte aligned (else one load all the same, which
+// the hardware takes from any element on)
+template <typename T, bool VEC>
+__device__ __forceinline__ typename Mfma<T>::vec_t load16(const T *p)
+{
+    typedef typename Mfma<T>::vec_t V;
+    if (VEC) return *(const V *)p;
+    const typename Mfma<T>::uvec_t u = *(const typename Mfma<T>::uvec_t *)p;
+    V v;
+    __builtin_memcpy(&v, &u, 16);
+    return v;
+}
+
 template <typename T, bool EDGE, int EPI>
 __device__ __forceinline__ void gemm_tile(const GemmDesc &g, const T *__restrict__ A, const T *__restrict__ B,
                                           T *__restrict__ C, int m0, int n0, int K,
@@ -152,7 +174,7 @@ struct Tile64Smem {
 
 // bscale (optional): row k of B is multiplied by bscale[k] as it is loaded,
 // one rounding, as a separately scaled copy of B would hold it
-template <typename T, bool EDGE, int EPI>
+template <typename T, bool EDGE, int EPI, bool VEC = true, bool DORD = false>
 __device__ __forceinline__ void gemm_tile64(const GemmDesc &g, const T *__restrict__ A, const T *__restrict__ B,
                                             T *__restrict__ C, int m0, int n0, int K, Tile64Smem<T> &sm,
                                             const T *__restrict__ bscale = nullptr)
@@ -177,8 +199,8 @@ __device__ __forceinline__ void gemm_tile64(const GemmDesc &g, const T *__restri
             const int ar = idx / ACH, ac = (idx % ACH) * EPV;
             const int br = idx / BCH, bc = (idx % BCH) * EPV;
             if (!EDGE) {
-                ra[it] = *(const V *)(A + (long)(m0 + ar) * lda + k0 + ac);
-                rb[it] = *(const V *)(B + (long)(k0 + br) * ldb + n0 + bc);
+                ra[it] = load16<T, VEC>(A + (long)(m0 + ar) * lda + k0 + ac);
+                rb[it] = load16<T, VEC>(B + (long)(k0 + br) * ldb + n0 + bc);
                 if (bscale) {
                     T *pb = (T *)&rb[it];
                     const T sc = bscale[k0 + br];
@@ -208,9 +230,9 @@ __device__ __forceinline__ void gemm_tile64(const GemmDesc &g, const T *__restri
             const int ar = idx / ACH, ac = (idx % ACH) * EPV;
             const T *pa = (const T *)&ra[it];
 #pragma unroll
-            for (int e = 0; e < EPV; e++) sm.As[buf][ar * AL + ac + e] = pa[e];
+            for (int e = 0; e < EPV; e++) sm.As[buf][ar * AL + k_place<DORD>(ac + e)] = pa[e];
             const int br = idx / BCH, bc = (idx % BCH) * EPV;
-            *(V *)&sm.Bs[buf][br * BT64 + bc] = rb[it];
+            *(V *)&sm.Bs[buf][k_place<DORD>(br) * BT64 + bc] = rb[it];
         }
     };
 
