@@ -211,8 +211,9 @@ struct IntC {
 
 // Per column step j (one grid-wide exchange):
 //   gather   every workgroup polls all words of all messages (the candidate
-//            row of every workgroup) and puts them into LDS: the threads' loads are all in flight at once, and a thread
-//            repeats its own until their tags are the step's;
+//            row of every workgroup) and puts them into LDS: the threads'
+//            loads are all in flight at once, and a thread repeats its own
+//            until their tags are the step's;
 //   reduce   each wavefront reduces the G candidates (largest |x|, lowest
 //            row on ties) -- identical result everywhere, no extra barrier;
 //   swap     the owners of rows j and p exchange rows, row j scaled by 1/d;
@@ -226,7 +227,7 @@ struct IntC {
 // device-coherent level, the reduction of the candidates, 1/d.  FP64, 16
 // columns, alone on the device, before and after the tagged messages, the
 // DPP reductions, the rotation and the copies of the current rows: 60 -> 30 us
-// for 256 rows, 60 -> 47 us for 1000 rows (one workgroup both now), 64.5 -> 48
+// for 256 rows (one workgroup), 60 -> 43.5 us for 4096 (16 of them), 64.5 -> 48
 // us for 9984 rows (39 workgroups), about 105 -> 61 us for 60000 rows; of the
 // 48 us, 2.8 us per column: 1.4 the wait for the other workgroups' messages,
 // 0.3 reduction and 1/d, 0.3 swap, 0.6 update, candidate and sending, the rest
@@ -238,6 +239,7 @@ struct LeafSmem {
         unsigned xch[2][LeafMsg<T, W>::XW];
     };
     alignas(16) unsigned pub[LeafMsg<T, W>::NW];   // the candidate before it is sent
+    alignas(16) T cur[W];                          // row j in the order of the messages, where it is the pivot row
     T top[W * W];                                  // rows c .. c+W-1 as they stand, in column order
     int top_lorig[W], top_borig[W];
     PivKey red[NTL / 64];
@@ -451,9 +453,9 @@ __device__ __forceinline__ void leaf_body(const LeafArgs<T> &a, const int bid, L
         const int p = none ? j : br;
         const unsigned *pslot = xb + bg * NW;
         if (none) {   // row j in the messages' order (every wavefront writes the same)
-            if (lane < W) ((T *)sm.pub)[lane] = sm.top[jl * W + (jl + lane) % W];
+            if (lane < W) sm.cur[lane] = sm.top[jl * W + (jl + lane) % W];
             wave_sync();
-            pslot = sm.pub;
+            pslot = (const unsigned *)sm.cur;
         }
 #pragma clang loop unroll(full)
         for (int k = 0; k < W; k++) us[k] = ((const T *)pslot)[k];

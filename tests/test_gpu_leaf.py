@@ -1,5 +1,5 @@
-"""The panel leaf at the edges of its launch shapes: one workgroup up to 1024
-rows (1, 2 or 4 rows per thread), several above; ties and columns without a
+"""The panel leaf at the edges of its launch shapes: one workgroup up to 512
+rows (1 or 2 rows per thread), several above; ties and columns without a
 comparable candidate decided as the oracle decides them."""
 import numpy as np
 import pytest
