@@ -95,22 +95,37 @@ __global__ __launch_bounds__(256) void rowperm_kernel(PermArgs<T> a)
     rowperm_strip<T>(a, blockIdx.x, (T *)smem_raw);
 }
 
-// pairs of the block's row permutation: (i+k, orig[i+k]) and (piv[i+k], orig[piv[i+k]])
-// The block-level permutation (lu2.c:524-556) without LDS staging, in two
+// The block-level permutation (lu2.c:524-556), pairs (i+k, orig[i+k]) and
+// (piv[i+k], orig[piv[i+k]]), without LDS staging, in two
 // launches over (pair, 1024-column chunk).  Destinations inside the block go
 // to the staging buffer W (scaled by 1/d), so pass 0 reads A and writes only
 // W.  A row below the block only ever receives content that started in the
 // block (content that enters the block from below stays there), so pass 1
 // reads block rows of A, which no pass writes, and writes rows below, which
 // pass 1 never reads.  Every read of a row below happens in pass 0.
+// first: the pairs are formed here from the block's pivots and origins (a
+// launch of its own before), and kept for the remaining columns.
 template <typename T>
-__global__ __launch_bounds__(256) void staged_perm_kernel(PermArgs<T> a, int pass)
+__global__ __launch_bounds__(256) void staged_perm_kernel(PermArgs<T> a, int pass, const int *piv, const int *orig,
+                                                          int *dst, int *src)
 {
     const int pr = blockIdx.y;
-    const int d = a.dst[pr];
+    int d, sr;
+    if (piv) {
+        const int nb = a.w1 - a.w0;
+        d = pr < nb ? a.w0 + pr : piv[a.w0 + pr - nb];
+        sr = orig[d];
+        if (blockIdx.x == 0 && pass == 0 && threadIdx.x == 0) {
+            dst[pr] = d;
+            src[pr] = sr;
+        }
+    } else {
+        d = a.dst[pr];
+        sr = a.src[pr];
+    }
     const bool to_w = (d >= a.w0 && d < a.w1);
     if (to_w != (pass == 0)) return;
-    const T *srow = a.A + (long)a.src[pr] * a.lda;
+    const T *srow = a.A + (long)sr * a.lda;
     const bool scale = (d >= a.d0 && d < a.d1);
     const T sc = scale ? a.invd[d] : T(1);
     T *drow = to_w ? a.W + (long)(d - a.w0) * a.ldw - a.c0 : a.A + (long)d * a.lda;
@@ -123,18 +138,6 @@ __global__ __launch_bounds__(256) void staged_perm_kernel(PermArgs<T> a, int pas
             if (scale && col < a.sce) v *= sc;
             drow[col] = v;
         }
-    }
-}
-
-__global__ void block_pairs_kernel(const int *piv, const int *orig, int i, int nb, int *dst, int *src)
-{
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < nb) {
-        dst[k] = i + k;
-        src[k] = orig[i + k];
-        const int p = piv[i + k];
-        dst[nb + k] = p;
-        src[nb + k] = orig[p];
     }
 }
 
@@ -666,10 +669,10 @@ struct Factor {
         if (W == 32 && rpt > 2) rpt = 2;
         if (W == 16 && rpt > 4) rpt = 4;
         if (rpt == 3) rpt = 4;
-        // as many rows as one workgroup's registers hold: no exchange through
-        // memory at all
-        const int rmax = (W == 16) ? 4 : 2;
-        if (R <= NTL * rmax) rpt = (R <= NTL) ? 1 : (R <= 2 * NTL) ? 2 : 4;
+        // up to 512 rows in one workgroup: no exchange through memory (above
+        // that four rows per thread would cost more: 1000 rows 47 us, and with
+        // the exchange 4096 rows take 43.5 us at one row per thread)
+        if (R <= 2 * NTL) rpt = (R <= NTL) ? 1 : 2;
         const int G = (R + NTL * rpt - 1) / (NTL * rpt);
         if (G > LEAF_GMAX) {
             lu2mi_set_error_msg("leaf: %d rows need %d workgroups (> %d)", R, G, LEAF_GMAX);
@@ -708,7 +711,7 @@ struct Factor {
     }
 
     int rowperm(const int *dst, const int *src, int np, int c0, int c1, int k0, int k1, int sce, int d0,
-                int d1, T *Wb, long ldw, int w0, int w1)
+                int d1, T *Wb, long ldw, int w0, int w1, bool first = false)
     {
         if (c1 <= c0) return LU2MI_OK;
         static bool lds_attr = false;
@@ -725,8 +728,10 @@ struct Factor {
             // block level: destinations in [w0, w1) are the block's rows
             p.sw = 0;
             const dim3 grid((c1 - c0 + 1023) / 1024, np);
-            hipLaunchKernelGGL(staged_perm_kernel<T>, grid, dim3(256), 0, ctx->stream, p, 0);
-            hipLaunchKernelGGL(staged_perm_kernel<T>, grid, dim3(256), 0, ctx->stream, p, 1);
+            for (int pass = 0; pass < 2; pass++)
+                hipLaunchKernelGGL(staged_perm_kernel<T>, grid, dim3(256), 0, ctx->stream, p, pass,
+                                   first ? (const int *)ctx->d_piv : nullptr, (const int *)ctx->d_orig, (int *)dst,
+                                   (int *)src);
             LU2MI_CHECK(hipGetLastError());
             return LU2MI_OK;
         }
@@ -892,18 +897,16 @@ struct Factor {
         set_block(i);
         int ts;
         LU2MI_TRY(tbegin(LU2MI_T_PANEL, ts));
-        hipLaunchKernelGGL(fill_kernel<T>, dim3(256), dim3(256), 0, ctx->stream, linv, (long)nb * nb, T(0));
-        LU2MI_CHECK(hipGetLastError());
         LU2MI_TRY(panel(i, i, nb));
         return tend(LU2MI_T_PANEL, ts, (double)(n - i) * nb * nb, 0.0);
     }
 
     // block-level row permutation of columns [c0, c1) with its timing
-    int block_perm(int i, int c0, int c1, T *wb, long ldw)
+    int block_perm(int i, int c0, int c1, T *wb, long ldw, bool first = false)
     {
         int ts;
         LU2MI_TRY(tbegin(LU2MI_T_SWAP, ts));
-        LU2MI_TRY(rowperm(pairs, pairs + 2 * nb, 2 * nb, c0, c1, 0, 0, n + 1, i, i + nb, wb, ldw, i, i + nb));
+        LU2MI_TRY(rowperm(pairs, pairs + 2 * nb, 2 * nb, c0, c1, 0, 0, n + 1, i, i + nb, wb, ldw, i, i + nb, first));
         return tend(LU2MI_T_SWAP, ts, 0.0, 32.0 * nb * (double)(c1 - c0));
     }
 
@@ -945,6 +948,14 @@ struct Factor {
         const bool la = ctx->lookahead != 0;
         hipStream_t s1 = ctx->stream;
         bool panel_pending = false;   // panel(i) issued on the second stream
+        // the inverses' blocks above the diagonal, which nothing writes, zeroed
+        // once for all blocks (a launch per block stood before every panel)
+        {
+            T *const z = linv_all ? linv_all : linv_base;
+            const long count = (long)nb * (linv_all ? n : 2 * nb);
+            hipLaunchKernelGGL(fill_kernel<T>, dim3(1024), dim3(256), 0, s1, z, count, T(0));
+            LU2MI_CHECK(hipGetLastError());
+        }
         LU2MI_TRY(start_panel(0));
         for (int i = 0; i < n; i += nb) {
             if (panel_pending) {
@@ -952,17 +963,13 @@ struct Factor {
                 panel_pending = false;
             }
             set_block(i);
-            int *const pairs_i = pairs;
             const int ncols = n + 1 - (i + nb);
             const int M = n - i - nb;
             const int na = (la && M > 0) ? nb : ncols;   // columns before the split
             // block-level row permutation over [i+nb, n], 1/d scaling of the
             // block rows, block rows staged in w (lu2.c:502-509 awork copy)
-            hipLaunchKernelGGL(block_pairs_kernel, dim3((nb + 255) / 256), dim3(256), 0, s1, ctx->d_piv,
-                               ctx->d_orig, i, nb, pairs_i, pairs_i + 2 * nb);
-            LU2MI_CHECK(hipGetLastError());
             const long ldw = (ncols + 3) & ~3L;   // 16-byte rows for FP64 and FP32
-            LU2MI_TRY(block_perm(i, i + nb, i + nb + na, wbuf, ldw));
+            LU2MI_TRY(block_perm(i, i + nb, i + nb + na, wbuf, ldw, true));
             // U12 = inv(D^-1 L11) * staged rows   (lu2.c:511-512)
             LU2MI_TRY(u12(i, i + nb, na, wbuf, ldw));
             if (M <= 0) continue;
