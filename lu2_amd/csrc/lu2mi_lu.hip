@@ -154,45 +154,55 @@ __global__ void scale_copy_kernel(const T *A, long lda, int r0, int c0, int h, i
 }
 
 // ---------------------------------------------------------------------------
-// Recursion nodes of half-width h <= 64, one workgroup (one 64x64 tile) per
-// step instead of two launches each; same arithmetic as the separate steps.
-// node_trsm64: X = inv(D^-1 L11) * (rows [c, c+h) of the right half scaled
-// by 1/d), the scaling done as the rows are loaded (the staging copy's
-// values); the tile reads all of its rows before it writes them back.
+// Recursion nodes of half-width h <= 64: one workgroup (one 64x64 tile) per
+// step, and the steps that follow one another in the recursion -- the inverse
+// blocks of the nodes that end at a leaf, deepest first, then the TRSM of the
+// node whose left half they close -- in one launch.  Same arithmetic as the
+// separate steps; what a launch costs is not its work (4-6 us each, of which
+// 1-2 us arithmetic) but being one more in the panel's chain.
+//   inverse block: X21 = -inv22 * (L21 * inv11), tmp passes between the
+//     products through memory
+//   TRSM: X = inv(D^-1 L11) * (rows [c, c+h) of the right half scaled by 1/d),
+//     the scaling done as the rows are loaded (the staging copy's values); the
+//     tile reads all of its rows before it writes them back
+struct NodeSteps {
+    int ninv;               // inverse blocks, at most one per half-width 16, 32, 64
+    int inv_c[3], inv_h[3];
+    int trsm_c, trsm_h;     // trsm_h = 0: none
+};
 template <typename T>
-__global__ __launch_bounds__(256) void node_trsm64_kernel(T *A, long lda, int c, int h, const T *linv, int ldl,
-                                                          long off, const T *invd)
+__global__ __launch_bounds__(256) void node_steps64_kernel(T *A, long lda, NodeSteps ns, T *linv, int ldl, int i,
+                                                           T *tmp, const T *invd)
 {
     using namespace lu2mi_gemm;
     __shared__ Tile64Smem<T> sm;
     __builtin_amdgcn_s_setprio(3);
+    auto fence = [&]() __attribute__((always_inline)) {
+        __threadfence();
+        __syncthreads();
+    };
     GemmDesc g;
-    g.M = h; g.N = h; g.K = h; g.alpha = 1.0; g.beta = 0.0;
-    g.lda = ldl; g.ldb = lda; g.ldc = lda; g.a_lower = 1;
-    T *X = A + (long)c * lda + c + h;
-    gemm_tile64<T, true, EPI_SET>(g, linv + off * ldl + off, X, X, 0, 0, h, sm, invd + c);
+    for (int q = 0; q < ns.ninv; q++) {
+        const int c = ns.inv_c[q], h = ns.inv_h[q];
+        const long off = c - i;
+        g.M = h; g.N = h; g.K = h; g.alpha = 1.0; g.beta = 0.0;
+        g.lda = lda; g.ldb = ldl; g.ldc = h; g.a_lower = 0;
+        gemm_tile64<T, true, EPI_SET>(g, A + (long)(c + h) * lda + c, linv + off * ldl + off, tmp, 0, 0, h, sm);
+        fence();
+        g.alpha = -1.0; g.lda = ldl; g.ldb = h; g.ldc = ldl; g.a_lower = 1;
+        gemm_tile64<T, true, EPI_GENERAL>(g, linv + (off + h) * ldl + off + h, tmp, linv + (off + h) * ldl + off, 0,
+                                          0, h, sm);
+        fence();
+    }
+    if (ns.trsm_h) {
+        const int c = ns.trsm_c, h = ns.trsm_h;
+        const long off = c - i;
+        g.M = h; g.N = h; g.K = h; g.alpha = 1.0; g.beta = 0.0;
+        g.lda = ldl; g.ldb = lda; g.ldc = lda; g.a_lower = 1;
+        T *X = A + (long)c * lda + c + h;
+        gemm_tile64<T, true, EPI_SET>(g, linv + off * ldl + off, X, X, 0, 0, h, sm, invd + c);
+    }
 }
-
-// node_inv64: the node's off-diagonal inverse block, X21 = -inv22 * (L21 * inv11),
-// both products in one workgroup (tmp passes between them through memory)
-template <typename T>
-__global__ __launch_bounds__(256) void node_inv64_kernel(const T *A, long lda, int c, int h, T *linv, int ldl,
-                                                         long off, T *tmp)
-{
-    using namespace lu2mi_gemm;
-    __shared__ Tile64Smem<T> sm;
-    __builtin_amdgcn_s_setprio(3);
-    GemmDesc g;
-    g.M = h; g.N = h; g.K = h; g.alpha = 1.0; g.beta = 0.0;
-    g.lda = lda; g.ldb = ldl; g.ldc = h; g.a_lower = 0;
-    gemm_tile64<T, true, EPI_SET>(g, A + (long)(c + h) * lda + c, linv + off * ldl + off, tmp, 0, 0, h, sm);
-    __threadfence();
-    __syncthreads();
-    g.alpha = -1.0; g.lda = ldl; g.ldb = h; g.ldc = ldl; g.a_lower = 1;
-    gemm_tile64<T, true, EPI_GENERAL>(g, linv + (off + h) * ldl + off + h, tmp, linv + (off + h) * ldl + off, 0, 0,
-                                      h, sm);
-}
-
 // column-major panel (m columns of ld rows, rows [r0, r0+R)) <-> row-major (R x ldp)
 __global__ void cm_to_rm_kernel(const double *cm, long ld, int r0, int R, int m, double *rm, long ldp, int back)
 {
@@ -817,6 +827,22 @@ struct Factor {
         return LU2MI_OK;
     }
 
+    NodeSteps steps{};   // inverse blocks due, not launched yet
+
+    // the inverse blocks due, and the TRSM of node (c, 2h) if h > 0
+    int node_steps(int i, int c, int h)
+    {
+        steps.trsm_c = c;
+        steps.trsm_h = h;
+        if (steps.ninv || h) {
+            hipLaunchKernelGGL(node_steps64_kernel<T>, dim3(1), dim3(256), 0, ctx->stream, A, lda, steps, linv, nb, i,
+                               tmp, Prec<T>::invd(ctx));
+            LU2MI_CHECK(hipGetLastError());
+        }
+        steps = NodeSteps{};
+        return LU2MI_OK;
+    }
+
     int panel(int i, int c, int w)
     {
         if (sub_ok(w)) return subpanel(i, c, w);
@@ -824,18 +850,16 @@ struct Factor {
         const int h = w / 2;
         LU2MI_TRY(panel(i, c, h));
         const long off = (long)(c - i);
-        if (h <= lu2mi_gemm::BT64) {   // one workgroup per step (see node_trsm64_kernel)
-            hipLaunchKernelGGL(node_trsm64_kernel<T>, dim3(1), dim3(256), 0, ctx->stream, A, lda, c, h, linv, nb, off,
-                               Prec<T>::invd(ctx));
-            LU2MI_CHECK(hipGetLastError());
+        if (h <= lu2mi_gemm::BT64) {   // one workgroup per step (see node_steps64_kernel)
+            LU2MI_TRY(node_steps(i, c, h));
             LU2MI_TRY(gemm_call<T>(ctx, n - c - h, h, h, -1.0, A + (long)(c + h) * lda + c, lda,
                                    A + (long)c * lda + c + h, lda, 1.0, A + (long)(c + h) * lda + c + h, lda, 0));
             LU2MI_TRY(panel(i, c + h, h));
-            hipLaunchKernelGGL(node_inv64_kernel<T>, dim3(1), dim3(256), 0, ctx->stream, A, lda, c, h, linv, nb, off,
-                               tmp);
-            LU2MI_CHECK(hipGetLastError());
+            steps.inv_c[steps.ninv] = c;
+            steps.inv_h[steps.ninv++] = h;
             return LU2MI_OK;
         }
+        LU2MI_TRY(node_steps(i, 0, 0));
         // right half of this node: rows [c, c+h) scaled by 1/d, then
         // X = inv(D^-1 L11) * scaled rows, then the rows below
         {
@@ -849,6 +873,7 @@ struct Factor {
                                    A + (long)c * lda + c + h, lda, 1.0, A + (long)(c + h) * lda + c + h, lda, 0));
         }
         LU2MI_TRY(panel(i, c + h, h));
+        LU2MI_TRY(node_steps(i, 0, 0));
         // off-diagonal block of the inverse: X21 = -inv22 * L21 * inv11
         {
             LU2MI_TRY(gemm_call<T>(ctx, h, h, h, 1.0, A + (long)(c + h) * lda + c, lda, linv + off * nb + off, nb,
@@ -898,6 +923,7 @@ struct Factor {
         int ts;
         LU2MI_TRY(tbegin(LU2MI_T_PANEL, ts));
         LU2MI_TRY(panel(i, i, nb));
+        LU2MI_TRY(node_steps(i, 0, 0));
         return tend(LU2MI_T_PANEL, ts, (double)(n - i) * nb * nb, 0.0);
     }
 
@@ -1104,6 +1130,7 @@ int lu2mi_cm_panel_f64(lu2mi_ctx *ctx, double *dcm, long ld, int n, int m, int i
     ctx->bar_count = 0;
     ctx->gbar_count = 0;
     if (rc == LU2MI_OK) rc = f.panel(0, 0, m);
+    if (rc == LU2MI_OK) rc = f.node_steps(0, 0, 0);
     if (rc == LU2MI_OK) {
         hipLaunchKernelGGL(cm_to_rm_kernel, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, ctx->stream, dcm, ld,
                            i, R, m, P, ldp, 1);
