@@ -187,9 +187,15 @@ static int launch_gemm(const GemmDesc &g, hipStream_t s)
     // tiles here too, in the K order of the tile they stand for (same bits).
     // n = 512 nb = 64 2.40 -> 2.20 ms, n = 2048 nb = 256 10.0 -> 9.55 ms (a
     // 128x128 U12 product of 256 columns there took 65 us), n = 9984 nb = 256
-    // 62.5 -> 59.9 ms.
-    if (vec && g.tag != 0 && g.batch == 1 && total < num_cu && (sizeof(T) == 4 || direct || g.tag == 2) &&
-        (g.a_lower ? epi == EPI_SET : epi == EPI_SUB)) {
+    // 62.5 -> 59.9 ms.  Against the direct-to-LDS tile only while a CU gets at
+    // most three 64x64 tiles, that is up to 3/4 of a large workgroup per CU
+    // (direct tile and 64x64 tiles at K = 512: 128 workgroups 86 and 64 us, 192
+    // 89 and 81, 208 90 and 97, 248 92 and 99; at K = 2048 192 274 and 248, 208
+    // 276 and 312); the register-staged tiles, FP64 and FP32, are slower than
+    // the 64x64 ones up to a tile per CU (FP32 K = 1024, 248: 115 and 109 us)
+    const long large = g.a_lower ? (long)((tiles_m + 1) / 2) * tiles_n : total;   // the large kernel's workgroups
+    if (vec && g.tag != 0 && g.batch == 1 && total < num_cu && !(direct && 4 * large > 3L * num_cu) &&
+        (sizeof(T) == 4 || direct || g.tag == 2) && (g.a_lower ? epi == EPI_SET : epi == EPI_SUB)) {
         const int tm64 = (g.M + BT64 - 1) / BT64, tn64 = (g.N + BT64 - 1) / BT64;
         dim3 grid64((unsigned)(tm64 * tn64)), block64(NT);
         constexpr bool DO = sizeof(T) == 8;
