@@ -21,7 +21,9 @@ using namespace lu2mi_gemm;
 // padding and spread over more workgroups; every element keeps the K range
 // of the 128x128 tile that contains it, so the results are the 128x128
 // kernel's bits.
-template <typename T, int EPI, bool VEC, bool DORD = false>
+// TAIL: for a K that ends within a stage (a kernel of its own: with both loops
+// in one the edge tiles, all there is of a narrow product, were 1-3% slower).
+template <typename T, int EPI, bool VEC, bool DORD = false, bool TAIL = false>
 __global__ __launch_bounds__(NT) void gemm64_kernel(GemmDesc g, int tiles_m, int tiles_n)
 {
     __shared__ Tile64Smem<T> sm;
@@ -32,8 +34,8 @@ __global__ __launch_bounds__(NT) void gemm64_kernel(GemmDesc g, int tiles_m, int
     const T *B = (const T *)g.B + bz * g.sB;
     T *C = (T *)g.C + bz * g.sC;
     const int K = g.a_lower ? min(g.K, (m0 & ~(BM - 1)) + BM) : g.K;
-    const bool interior = (m0 + BT64 <= g.M) && (n0 + BT64 <= g.N) && (K % Mfma<T>::BK == 0);
-    if (interior) gemm_tile64<T, false, EPI, VEC, DORD>(g, A, B, C, m0, n0, K, sm);
+    const bool interior = (m0 + BT64 <= g.M) && (n0 + BT64 <= g.N) && (TAIL || K % Mfma<T>::BK == 0);
+    if (interior) gemm_tile64<T, false, EPI, VEC, DORD, TAIL>(g, A, B, C, m0, n0, K, sm);
     else gemm_tile64<T, true, EPI, VEC, DORD>(g, A, B, C, m0, n0, K, sm);
 }
 
@@ -162,9 +164,13 @@ static int launch_gemm(const GemmDesc &g, hipStream_t s)
     // column) run the 64x64 tiles with unaligned 16-byte loads, in one general
     // form (element loads with bounds checks in 128x128 tiles before: at an odd
     // stride 700 x 900 x 300 80 -> 40 us, 40 x 8000 x 100 43 -> 28 us,
-    // 3000 x 3000 x 1000 473 -> 392 us), and above the 64x64 tiles' sizes the
+    // 3000 x 3000 x 1500 674 -> 493 us), and above the 64x64 tiles' sizes the
     // 128x128 tiles with element loads (6001 x 6001 x 513 806 us, 822 with
-    // unaligned ones)
+    // unaligned ones).  A K that ends within a stage costs one checked stage
+    // (TAIL): with bounds checks in every stage the 64x64 tiles were slower
+    // than the 128x128 ones wherever those fill their last round of CUs (FP32
+    // 5700 x 5700 x 2047 128x128 tiles 1456 us, 64x64 with checks throughout
+    // 1834, with TAIL 1305; FP64 3450 x 3450 x 701 340, 354, 328)
     constexpr long EPV = Mfma<T>::EPV;
     const bool vec = aligned16(g.A) && aligned16(g.B) && (g.lda % EPV == 0) && (g.ldb % EPV == 0) &&
                      (g.sA % EPV == 0) && (g.sB % EPV == 0);
@@ -213,7 +219,10 @@ static int launch_gemm(const GemmDesc &g, hipStream_t s)
     if (g.tag == 0 && (g.M <= BT64 || g.N <= BT64 || underfilled)) {
         const int tm64 = (g.M + BT64 - 1) / BT64, tn64 = (g.N + BT64 - 1) / BT64;
         dim3 grid64((unsigned)(tm64 * tn64), (unsigned)g.batch), block64(NT);
-        if (!vec)
+        if (!vec && g.K % Mfma<T>::BK != 0 && g.M >= BT64 && g.N >= BT64)
+            hipLaunchKernelGGL((gemm64_kernel<T, EPI_GENERAL, false, false, true>), grid64, block64, 0, s, g, tm64,
+                               tn64);
+        else if (!vec)
             hipLaunchKernelGGL((gemm64_kernel<T, EPI_GENERAL, false>), grid64, block64, 0, s, g, tm64, tn64);
         else if (epi == EPI_SUB)
             hipLaunchKernelGGL((gemm64_kernel<T, EPI_SUB, true>), grid64, block64, 0, s, g, tm64, tn64);

@@ -174,7 +174,8 @@ struct Tile64Smem {
 
 // bscale (optional): row k of B is multiplied by bscale[k] as it is loaded,
 // one rounding, as a separately scaled copy of B would hold it
-template <typename T, bool EDGE, int EPI, bool VEC = true, bool DORD = false>
+// TAIL (interior tiles): any K >= 1; the last stage is loaded element by element
+template <typename T, bool EDGE, int EPI, bool VEC = true, bool DORD = false, bool TAIL = false>
 __device__ __forceinline__ void gemm_tile64(const GemmDesc &g, const T *__restrict__ A, const T *__restrict__ B,
                                             T *__restrict__ C, int m0, int n0, int K, Tile64Smem<T> &sm,
                                             const T *__restrict__ bscale = nullptr)
@@ -260,13 +261,52 @@ __device__ __forceinline__ void gemm_tile64(const GemmDesc &g, const T *__restri
     };
 
     const int nk = (K + BKT - 1) / BKT;
-    if (nk > 0) {
-        load_tiles(0);
+    if (!TAIL) {
+        if (nk > 0) {
+            load_tiles(0);
+            store_tiles(0);
+            __syncthreads();
+            for (int kt = 0; kt < nk - 1; kt++) {
+                const int cur = kt & 1;
+                load_tiles((kt + 1) * BKT);
+                compute(cur);
+                store_tiles(cur ^ 1);
+                __syncthreads();
+            }
+            compute((nk - 1) & 1);
+        }
+    } else {
+        auto load_last = [&]() {
+            const int k0 = (nk - 1) * BKT;
+#pragma unroll
+            for (int it = 0; it < LPT; it++) {
+                const int idx = t + it * NT;
+                const int ar = idx / ACH, ac = (idx % ACH) * EPV;
+                const int br = idx / BCH, bc = (idx % BCH) * EPV;
+                T va[EPV], vb[EPV];
+#pragma unroll
+                for (int e = 0; e < EPV; e++) {
+                    va[e] = (k0 + ac + e < K) ? A[(long)(m0 + ar) * lda + k0 + ac + e] : T(0);
+                    vb[e] = (k0 + br < K) ? B[(long)(k0 + br) * ldb + n0 + bc + e] : T(0);
+                }
+                ra[it] = *(V *)va;
+                rb[it] = *(V *)vb;
+            }
+        };
+        if (nk > 1) load_tiles(0);
+        else load_last();
         store_tiles(0);
         __syncthreads();
-        for (int kt = 0; kt < nk - 1; kt++) {
+        for (int kt = 0; kt < nk - 2; kt++) {
             const int cur = kt & 1;
             load_tiles((kt + 1) * BKT);
+            compute(cur);
+            store_tiles(cur ^ 1);
+            __syncthreads();
+        }
+        if (nk > 1) {
+            const int cur = nk & 1;   // stage nk - 2's buffer
+            load_last();
             compute(cur);
             store_tiles(cur ^ 1);
             __syncthreads();
