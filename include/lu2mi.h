@@ -56,10 +56,14 @@ extern "C" {
                                      registers; the two sum each product's K terms in
                                      different orders */
 #define LU2MI_OPT_DGEMM_TRAILING 7 /* 1: lu2mi_dgemm_dev (and lu2mi_sgemm_dev) run their
-                                     product with the trailing-update kernel (to measure or
-                                     test that kernel alone);
-                                     2: the same, with A taken as lower triangular (the U12
-                                     product's form: entries above the diagonal are not read) */
+                                     product as a trailing update of its size: with the
+                                     trailing-update kernel (to measure or test it) from one
+                                     128 x 128 tile per CU on, and below, as the
+                                     factorization does, in 64 x 64 tiles where those are
+                                     faster (same bits);
+                                     2: lu2mi_dgemm_dev the same, with A taken as lower
+                                     triangular (the U12 product's form: tiles above the
+                                     diagonal are not read) */
 #define LU2MI_OPT_STRICT_SYNC 8   /* 1: the back substitution publishes its cross-workgroup
                                      data with agent-scope release/acquire (an L2 writeback
                                      and invalidate per publication); default 0:

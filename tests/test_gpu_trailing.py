@@ -10,8 +10,8 @@ import lu2_amd as L
 
 pytestmark = pytest.mark.gpu
 
-# 18 x 17 tiles of 128x128, more than the device's 256 CUs
-RAGGED = (2200, 2111)
+# 18 x 17 tiles of 128x128, more than the device's 256 CUs, ragged and whole
+RAGGED, WHOLE = (2200, 2111), (2304, 2176)
 FORMS = [("f64", 1), ("f64", 0), ("f32", 1)]
 
 
@@ -53,6 +53,16 @@ def operands(form, m, n, k, seed):
     return tuple(rng.standard_normal(s).astype(dtype) for s in ((m, k), (k, n), (m, n)))
 
 
+def check_bound(form, got, a, b, c):
+    """|C - fl(C - AB)| <= gamma_{K+2} (|A||B| + |C|), the reference itself
+    rounded in FP64."""
+    u = 2.0 ** -53 if form[0] == "f64" else 2.0 ** -24
+    k = a.shape[1]
+    gamma = (k + 2) * u / (1 - (k + 2) * u)
+    a, b, c = (x.astype(np.float64) for x in (a, b, c))
+    assert np.all(np.abs(got - (c - a @ b)) <= 2 * gamma * (np.abs(a) @ np.abs(b) + np.abs(c)))
+
+
 @pytest.mark.parametrize("form", FORMS)
 @pytest.mark.parametrize("k", [40, 96])
 @pytest.mark.parametrize("m,n", [(64, 64), (130, 66), (1, 300), (1536, 2048), (1664, 2047), (1920, 2176)])
@@ -66,3 +76,44 @@ def test_trailing_bits_do_not_depend_on_the_tile(ctx, form, k, m, n):
     last = product(ctx, form, np.ascontiguousarray(a[-m:]), np.ascontiguousarray(b[:, -n:]),
                    np.ascontiguousarray(c[-m:, -n:]))
     assert np.array_equal(large[-m:, -n:], last)
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("k", [40, 96])
+def test_large_tiles_edge_and_interior(ctx, form, k):
+    """The large tiles' bounds-checked loads do the arithmetic of their
+    unchecked ones: a ragged product against one whose tiles are all interior
+    (K filled up to whole stages with zeros)."""
+    a, b, c = operands(form, *WHOLE, k, k + 1)
+    a, b = padded(a, WHOLE[0], -(-k // 32) * 32, a.dtype), padded(b, -(-k // 32) * 32, WHOLE[1], b.dtype)
+    whole = product(ctx, form, a, b, c)
+    m, n = RAGGED
+    ragged = product(ctx, form, np.ascontiguousarray(a[:m, :k]), np.ascontiguousarray(b[:k, :n]),
+                     np.ascontiguousarray(c[:m, :n]))
+    assert np.array_equal(whole[:m, :n], ragged)
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("k", [17, 512])
+def test_large_tiles_error_bound(ctx, form, k):
+    a, b, c = operands(form, *RAGGED, k, k + 2)
+    check_bound(form, product(ctx, form, a, b, c), a, b, c)
+
+
+@pytest.mark.parametrize("kernel", [1, 0])
+def test_u12_edge_interior_and_small(ctx, kernel):
+    """The U12 product, A lower triangular, C not read: 8 x 33 large tiles,
+    ragged and whole, within the product's error bound, and its first rows and
+    columns as a product of their own in 64x64 tiles."""
+    form, m, n = ("f64", kernel), 1000, 4200
+    a, b, _ = operands(form, m, n, m, 3)
+    a = np.tril(a)
+    nan = np.full((1024, 4224), np.nan)
+    ragged = product(ctx, form, a, b, nan[:m, :n], lower=True)
+    check_bound(form, -ragged, a, b, np.zeros((m, n)))
+    whole = product(ctx, form, padded(a, 1024, 1024, np.float64), padded(b, 1024, 4224, np.float64), nan, lower=True)
+    assert np.array_equal(whole[:m, :n], ragged)
+    for mm, nn in ((64, 64), (130, 66), (1, 300), (500, 4200)):
+        small = product(ctx, form, np.ascontiguousarray(a[:mm, :mm]), np.ascontiguousarray(b[:mm, :nn]), nan[:mm, :nn],
+                        lower=True)
+        assert np.array_equal(ragged[:mm, :nn], small)
