@@ -161,7 +161,9 @@ static int launch_gemm(const GemmDesc &g, hipStream_t s)
         return LU2MI_ERR_ARG;
     }
     // 16-byte aligned rows of A and B; others (an odd row stride or first
-    // column) run the 64x64 tiles with unaligned 16-byte loads, in one general
+    // column), trailing updates apart (tag != 0: a factored matrix with an odd
+    // row stride keeps the 128x128 tiles with element loads at every size),
+    // run the 64x64 tiles with unaligned 16-byte loads, in one general
     // form (element loads with bounds checks in 128x128 tiles before: at an odd
     // stride 700 x 900 x 300 80 -> 40 us, 40 x 8000 x 100 43 -> 28 us,
     // 3000 x 3000 x 1500 674 -> 493 us), and above the 64x64 tiles' sizes the

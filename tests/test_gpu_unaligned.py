@@ -1,7 +1,9 @@
-"""Products on rows that are not 16-byte aligned, in FP64 and FP32: the bits
-of the same product on aligned rows, for every remainder of K."""
+"""Products and factorizations on rows that are not 16-byte aligned: the bits
+of the same on aligned rows."""
 import numpy as np
 import pytest
+
+import lu2_amd as L
 
 pytestmark = pytest.mark.gpu
 
@@ -45,3 +47,23 @@ def test_unaligned_products_any_k(ctx, prec, m, n, k):
         gamma = (k + 2) * u / (1 - (k + 2) * u)
         assert np.all(np.abs(got - (alpha * (a64 @ b64) + cc)) <= 2 * gamma * (np.abs(a64) @ np.abs(b64) + np.abs(cc)))
         assert np.array_equal(got, product(ctx, ap, bp, c0, alpha, beta, 0))
+
+
+@pytest.mark.parametrize("n,nb", [(64, 32), (544, 32), (1024, 128), (2048, 256)])
+def test_lu_odd_row_stride(ctx, oracle, n, nb):
+    """A matrix of n + 1 columns without padding.  Its trailing updates run in
+    the register-staged tiles, so its factors are those of the aligned matrix
+    with these tiles chosen."""
+    a0 = oracle.randomsetmat(n, n, n + 1)
+    even = np.zeros((n, n + 16))
+    even[:, :n + 1] = a0
+    x, piv, f = L.solve(a0, nb, L.PIV_GEPP, ctx)
+    ctx.set_option(L.OPT_TRAIL_KERNEL, 0)
+    try:
+        xe, pe, fe = L.solve(even, nb, L.PIV_GEPP, ctx)
+    finally:
+        ctx.set_option(L.OPT_TRAIL_KERNEL, 1)   # the library default
+    assert np.array_equal(piv, pe) and np.array_equal(x, xe) and np.array_equal(f, fe[:, :n + 1])
+    xo, po, _ = oracle.lumcolumn(a0, nb, oracle.PIV_GEPP)
+    assert np.array_equal(piv, po)
+    assert np.abs(x - xo).max() <= 1e-10 * np.abs(xo).max()
