@@ -8,7 +8,7 @@
 
 // ---------------------------------------------------------------------------
 // Leaf factorization: persistent kernel over rows [c, n), W columns; all
-// workgroups are co-resident and meet at a grid barrier once per column.
+// workgroups are co-resident and exchange messages once per column.
 namespace {
 constexpr int NTL = 256;        // threads per workgroup in the leaf kernel
 constexpr int LEAF_GMAX = 128;  // most workgroups a leaf launch may use
@@ -592,7 +592,10 @@ __device__ __forceinline__ void leaf_body(const LeafArgs<T> &a, const int bid, L
 }
 
 // at most 256 VGPRs for the 16-wide leaf, so that it fits on a SIMD beside one
-// wavefront of the trailing update
+// wavefront of the trailing update.  Within them (FP64) one row per thread
+// takes 146, two 209; four, for more than 32768 rows, spill 34 (140 bytes of
+// scratch a lane): 61 us a leaf at 60000 rows all the same, where the kernel
+// before the tagged messages took 105 with 220 VGPRs and no scratch
 template <typename T, int W, int RPT>
 __global__ __launch_bounds__(NTL, W == 16 ? 2 : 1) void leaf_kernel(LeafArgs<T> a)
 {

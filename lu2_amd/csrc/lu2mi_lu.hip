@@ -8,9 +8,9 @@
 //  per nb-block i:
 //    panel(i, nb)                       recursive halving down to a W-column leaf
 //      leaf   : one persistent kernel factors W columns of rows [c, n) held in
-//               registers; one grid barrier per column exchanges the
-//               per-workgroup pivot candidates (wavefront argmax, lowest row
-//               on ties) together with the candidate rows, so the winning row
+//               registers; one exchange per column brings every workgroup
+//               the pivot candidates of all (wavefront argmax, lowest row on
+//               ties) together with the candidate rows, so the winning row
 //               arrives with the decision.  It also forms the leaf's W x W
 //               block of (D^-1 L11)^-1.
 //      rowperm: the leaf's swaps applied to the other panel columns, with
@@ -158,8 +158,10 @@ __global__ void scale_copy_kernel(const T *A, long lda, int r0, int c0, int h, i
 // step, and the steps that follow one another in the recursion -- the inverse
 // blocks of the nodes that end at a leaf, deepest first, then the TRSM of the
 // node whose left half they close -- in one launch.  Same arithmetic as the
-// separate steps; what a launch costs is not its work (4-6 us each, of which
-// 1-2 us arithmetic) but being one more in the panel's chain.
+// separate steps; what a launch costs is not its work (a step of its own 4-6
+// us, of which 1-2 us arithmetic; together, alone on the device, 3.5 us for
+// one TRSM to 29 us for three inverse blocks and a TRSM, 10.4 us on average)
+// but being one more in the panel's chain.
 //   inverse block: X21 = -inv22 * (L21 * inv11), tmp passes between the
 //     products through memory
 //   TRSM: X = inv(D^-1 L11) * (rows [c, c+h) of the right half scaled by 1/d),
@@ -700,12 +702,13 @@ struct Factor {
         if (W == 32) fn = (rpt == 1) ? (const void *)leaf_kernel<T, 32, 1> : (const void *)leaf_kernel<T, 32, 2>;
         else fn = (rpt == 1) ? (const void *)leaf_kernel<T, 16, 1>
                  : (rpt == 2) ? (const void *)leaf_kernel<T, 16, 2> : (const void *)leaf_kernel<T, 16, 4>;
-        // All G workgroups must be resident together (they meet at the grid
-        // barrier).  An ordinary launch on an otherwise idle device places
-        // them all when occupancy allows it; the runtime's cooperative launch
-        // is not used because it holds a per-device resource that a second
-        // process on the same GPU cannot get.  The barrier's bounded spin
-        // turns any shortfall into LU2MI_ERR_DEVICE rather than a hang.
+        // All G workgroups must be resident together (each waits for the
+        // messages of all, once per column).  An ordinary launch on an
+        // otherwise idle device places them all when occupancy allows it; the
+        // runtime's cooperative launch is not used because it holds a
+        // per-device resource that a second process on the same GPU cannot
+        // get.  The wait's bounded spin turns any shortfall into
+        // LU2MI_ERR_DEVICE rather than a hang.
         int per_cu = 0;
         LU2MI_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, NTL, 0));
         if ((long)per_cu * ctx->num_cu < G) {
